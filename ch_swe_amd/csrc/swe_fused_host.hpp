@@ -79,16 +79,7 @@ inline int build_fused_tables(int N, int TY, FusedTables &ft, std::string &err, 
         return 1;
     ft.ntiles = 6 * ft.ntx * ft.nty;
     ft.segs.clear();
-    for (int p = 0; p < 6; p++)
-        for (int side = 0; side < 4; side++) {
-            // records segments: uniform pieces of at most R_SEG points, the
-            // extents a records frame holds
-            const int cnt = (n + R_SEG - 1) / R_SEG;
-            for (int k = 0; k < cnt; k++) {
-                const int lo = 1 + k * R_SEG, hi = std::min(n, lo + R_SEG - 1);
-                ft.segs.push_back(make_int4(p, side, lo, hi));
-            }
-        }
+    for (int i = 0; i < edge_blocks(N); i++) ft.segs.push_back(segment_of<0>(N, i));
     ft.nseg = (int)ft.segs.size();
     return tiling_fits(n, TY, ft, err) ? 0 : 1;
 }

@@ -189,9 +189,13 @@ __global__ void k_sync_weights(int N, double hx, T *qb, T *qt, T *ql, T *qr)
 }
 
 // panel-independent coefficient tables for the fused path (FP64 arithmetic,
-// stored in T) on the (N+1) x (N+1) index grid, plus f J^2 per panel
+// stored in T) on the (N+1) x (N+1) index grid, plus f J^2 per panel.  J Qi11
+// at the u points and J Qi22 at the v points: the flux J ut = J Qi11 u + ..
+// is formed first and ut = (J ut) / J from it, two coefficients per point
+// where Qi11, 1 / J and J are three.  (Two slots of the argument list are
+// unused.)
 template <typename T>
-__global__ void k_coef(int N, GeomParams g, T *JQ12, T *iJa, T *Q11, T *iJu, T *Ju, T *Q22, T *iJv, T *Jv, T *fJ2)
+__global__ void k_coef(int N, GeomParams g, T *JQ12, T *iJa, T *JQ11, T *iJu, T *, T *JQ22, T *iJv, T *, T *fJ2)
 {
     const int n = N + 1;
     long k = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -228,15 +232,17 @@ __global__ void k_coef(int N, GeomParams g, T *JQ12, T *iJa, T *Q11, T *iJu, T *
     iJa[r] = T(1.0 / (J * g.radius * g.hx));
     if (i <= N) {
         metric(0.5, 0.0, J, q11, q12, q22, X, Y, s);
-        Q11[r] = T(q11);
+        JQ11[r] = T(J * q11);
         iJu[r] = T(1.0 / J);
-        Ju[r] = T(J);
+    } else {
+        JQ11[r] = iJu[r] = T(0);
     }
     if (j <= N) {
         metric(0.0, 0.5, J, q11, q12, q22, X, Y, s);
-        Q22[r] = T(q22);
+        JQ22[r] = T(J * q22);
         iJv[r] = T(1.0 / J);
-        Jv[r] = T(J);
+    } else {
+        JQ22[r] = iJv[r] = T(0);
     }
 }
 

@@ -745,7 +745,6 @@ struct Engine : EngineBase {
     Coef<T> cf{};
     T *rec[2] = {nullptr, nullptr};
     int ntx = 0, nty = 0, ntiles = 0, nseg = 0, fwx = 0, fwy = 0;
-    int nthr = F_THREADS;  // workgroup size of the fused kernels
 
     size_t elem() const override { return sizeof(T); }
     bool fused() const override { return use_fused; }
@@ -825,7 +824,6 @@ struct Engine : EngineBase {
         // sbp63 runs on the multi-kernel path (the fused kernels' regions are
         // sized for the sbp21 / sbp42 closures)
         use_fused = !(p->cfg.flags & SWE_FLAG_UNFUSED) && order != 63;
-        nthr = p->cfg.block_threads ? p->cfg.block_threads : F_THREADS;
         if ((rc = alloc((void **)&part, 3 * INT_MAX_BLOCKS * sizeof(double))) ||
             (rc = alloc((void **)&red, 4 * sizeof(double))) ||
             (rc = alloc((void **)&dpart, (size_t)DIAG_K * INT_MAX_BLOCKS * sizeof(double))) ||
@@ -877,9 +875,9 @@ struct Engine : EngineBase {
         const int N = d.N, n = N + 1;
         int rc;
         // coefficient tables
-        T *tabs[8];
-        for (auto &t : tabs)
-            if ((rc = alloc((void **)&t, (size_t)n * n * sizeof(T)))) return rc;
+        T *tabs[8] = {};
+        for (T *&t : tabs)
+            if (&t != &tabs[4] && &t != &tabs[7] && (rc = alloc((void **)&t, (size_t)n * n * sizeof(T)))) return rc;
         T *tf;
         if ((rc = alloc((void **)&tf, 6 * (size_t)n * n * sizeof(T)))) return rc;
         k_coef<T><<<blocks_for(6L * n * n), TPB, 0, pl->stream>>>(N, g, tabs[0], tabs[1], tabs[2], tabs[3], tabs[4],
@@ -933,6 +931,7 @@ struct Engine : EngineBase {
         a.fwy = fwy;
         a.order = O;
         a.xcd = (pl->cfg.flags & SWE_FLAG_LINEAR_BLOCKS) ? 0 : 1;
+        a.rows = march_rows<T>(d.N + 1);
         a.general = (pl->cfg.flags & SWE_FLAG_GENERAL_TILES) ? 1 : 0;
         return a;
     }
@@ -950,7 +949,7 @@ struct Engine : EngineBase {
         StageArgs<T> a = stage_args<O>(in);
         a.out = out;
         a.rec_in = rec[0];
-        timer.launch(k_stage<T, O, TY, 0>, ntiles, nthr, pl->stream, 0, a);
+        timer.launch(k_stage<T, O, TY, 0>, stage_blocks(d.N, a.rows), F_STAGE_THREADS, pl->stream, 0, a);
     }
 
     // nsteps RK4 steps, each: records of v0, then the four stages, each
@@ -978,10 +977,10 @@ struct Engine : EngineBase {
                 a.a_dt = T(A[st]);
                 a.b_dt = T(B[st]);
                 a.rec_in = rec[st & 1];
-                if (st == 0) timer.launch(k_stage<T, O, TY, 1>, ntiles, nthr, pl->stream, 0, a);
-                else if (st == 3 && cmp) timer.launch(k_stage<T, O, TY, 4>, ntiles, nthr, pl->stream, 0, a);
-                else if (st == 3) timer.launch(k_stage<T, O, TY, 3>, ntiles, nthr, pl->stream, 0, a);
-                else timer.launch(k_stage<T, O, TY, 2>, ntiles, nthr, pl->stream, 0, a);
+                if (st == 0) timer.launch(k_stage<T, O, TY, 1>, stage_blocks(d.N, a.rows), F_STAGE_THREADS, pl->stream, 0, a);
+                else if (st == 3 && cmp) timer.launch(k_stage<T, O, TY, 4>, stage_blocks(d.N, a.rows), F_STAGE_THREADS, pl->stream, 0, a);
+                else if (st == 3) timer.launch(k_stage<T, O, TY, 3>, stage_blocks(d.N, a.rows), F_STAGE_THREADS, pl->stream, 0, a);
+                else timer.launch(k_stage<T, O, TY, 2>, stage_blocks(d.N, a.rows), F_STAGE_THREADS, pl->stream, 0, a);
                 if (st < 3) launch_records<O>(nexts[st], rec[(st + 1) & 1]);
             }
         }
@@ -2090,14 +2089,6 @@ int check_tables_ty(int N)
         const int4 a = segment_of<TY>(N, i), b = ft.segs[i];
         if (a.x != b.x || a.y != b.y || a.z != b.z || a.w != b.w)
             return fail(SWE_EINVAL, "edge segment decode disagrees with the segment table");
-    }
-    // every segment's band fits the records kernels' frame
-    for (int i = 0; i < ft.nseg; i++) {
-        const int4 g = ft.segs[i];
-        RTile<float> rt;
-        rt.setup(N, g.x, g.y, g.z, g.w, nullptr);
-        if (rt.frame_points() > RSmem<float>::CAP || rt.frame_points() > RTile<float>::CH * F_REC_THREADS)
-            return fail(SWE_EINVAL, "an edge segment's band exceeds the records frame");
     }
     // the launch order is a bijection of the tiles, side tiles first
     const int nt = ft.ntiles, e = side_tiles(ft.ntx, ft.nty);
