@@ -302,6 +302,7 @@ __global__ void k_dot_final(const double *part, int nb, double *out)
 {
     const int l = threadIdx.x & 63;
     double s = 0;
+#pragma unroll 8
     for (int b = l; b < nb; b += 64) s += part[b];
     for (int m = 32; m >= 1; m >>= 1) s += __shfl_down(s, m);
     if (threadIdx.x == 0) *out = s;
@@ -403,6 +404,7 @@ __global__ void k_reduce_final(const double *part, int nb, double *out)
 {
     const int l = threadIdx.x & 63;
     double s[3] = {0, 0, 0};
+#pragma unroll 8
     for (int k = l; k < nb; k += 64)
         for (int q = 0; q < 3; q++) s[q] += part[3 * k + q];
     for (int q = 0; q < 3; q++)
