@@ -320,42 +320,94 @@ __global__ void k_fill(double *p, int n, double v)
 // After convergence the update kernels do nothing, so x stays the iterate
 // that met the tolerance whatever iterations follow in the same batch.
 
-// x += alpha p, r -= alpha Ap, alpha = |r|^2 / (p, Ap) with |r| = sqrt(*rr)
-template <typename T>
-__global__ void k_cg_step(long n, T *x, T *r, const T *p, const T *Ap, const double *rr, const double *pap,
-                          const double *st)
+// An iteration after its two applies is three launches, each ending in partial
+// sums that every block of the next one adds up for itself.  At N = 96 a launch
+// costs 1.5 us and its gap whatever it does; as axpy, dot, final sum, step,
+// dot, final sum, check and direction (with a copy before the applies) an
+// iteration took 54 us, so 37.  The loops run over the padded fields, whose
+// padding has weight 0 (no index division).
+constexpr int CG_BLOCKS = 256, CG_TPB = 512;
+
+// the block's sum of s, in a fixed order, to every thread
+__device__ inline double cg_block_sum(double s, double (&ws)[CG_TPB / 64])
 {
-    const long k = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (k >= n || st[0] != 0.0) return;
-    const double rn = sqrt(*rr), alpha = rn * rn / *pap;
-    x[k] = x[k] + T(alpha) * p[k];
-    r[k] = r[k] + T(-alpha) * Ap[k];
+    for (int m = 32; m >= 1; m >>= 1) s += __shfl_down(s, m);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = s;
+    __syncthreads();
+    double r = ws[0];
+    for (int k = 1; k < CG_TPB / 64; k++) r += ws[k];
+    return r;
+}
+__device__ inline double cg_total(const double *part, double (&ws)[CG_TPB / 64])
+{
+    return cg_block_sum(threadIdx.x < CG_BLOCKS ? part[threadIdx.x] : 0.0, ws);
 }
 
-// the relative residual of iteration it against the tolerance (one thread)
-__global__ void k_cg_check(const double *rr_new, const double *bb, double rel_tol, double *st)
+// Ap = z + g t, partial sums of (z, Ap)
+template <typename T>
+__global__ __launch_bounds__(CG_TPB) void k_cg_ap(long n, const double *w, const T *z, const T *t, T g, T *Ap, double *part)
 {
-    if (threadIdx.x != 0 || st[0] != 0.0) return;
-    // st[3] counts the iterations, so that every batch of iterations is the
-    // same launch sequence (replayed from one graph)
-    const double it = st[3] + 1.0;
-    st[3] = it;
-    const double rel = sqrt(*rr_new) / sqrt(*bb);
-    st[2] = rel;
-    if (rel < rel_tol) {
-        st[0] = 1.0;
-        st[1] = it;
+    __shared__ double ws[CG_TPB / 64];
+    double s = 0;
+    for (long k = blockIdx.x * (long)CG_TPB + threadIdx.x; k < n; k += (long)CG_BLOCKS * CG_TPB) {
+        const T a = T(1.0) * z[k] + g * t[k];
+        const double wk = w[k];
+        Ap[k] = a;
+        if (wk != 0.0) s += wk * (double)z[k] * (double)a;
     }
+    s = cg_block_sum(s, ws);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// p = r + beta p, beta = (|r_new| / |r_old|)^2
+// x += alpha p, r -= alpha Ap, alpha = |r|^2 / (p, Ap) with |r| = sqrt(*rr);
+// partial sums of the new (r, r)
 template <typename T>
-__global__ void k_cg_dir(long n, T *p, const T *r, const double *rr_new, const double *rr_old, const double *st)
+__global__ __launch_bounds__(CG_TPB) void k_cg_step(long n, const double *w, T *x, T *r, const T *p, const T *Ap,
+                                                    const double *rr, const double *pap, const double *st, double *part)
 {
-    const long k = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (k >= n || st[0] != 0.0) return;
-    const double q = sqrt(*rr_new) / sqrt(*rr_old), beta = q * q;
-    p[k] = T(1.0) * r[k] + T(beta) * p[k];
+    __shared__ double ws[CG_TPB / 64];
+    if (st[0] != 0.0) return;
+    const double rn = sqrt(*rr), alpha = rn * rn / cg_total(pap, ws);
+    double s = 0;
+    for (long k = blockIdx.x * (long)CG_TPB + threadIdx.x; k < n; k += (long)CG_BLOCKS * CG_TPB) {
+        x[k] = x[k] + T(alpha) * p[k];
+        const T q = r[k] + T(-alpha) * Ap[k];
+        const double wk = w[k];
+        r[k] = q;
+        if (wk != 0.0) s += wk * (double)q * (double)q;
+    }
+    s = cg_block_sum(s, ws);
+    if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+// p = r + beta p, beta = (|r_new| / |r_old|)^2; block 0 keeps |r_new|^2 and
+// holds the relative residual against the tolerance.  (A block that comes late
+// may see the convergence it finds: p is not used any more then.)
+template <typename T>
+__global__ __launch_bounds__(CG_TPB) void k_cg_dir(long n, T *p, const T *r, const double *part, const double *rr_old,
+                                                   double *rr_new, const double *bb, double rel_tol, double *st)
+{
+    __shared__ double ws[CG_TPB / 64];
+    __shared__ double over;
+    if (threadIdx.x == 0) over = st[0];
+    __syncthreads();
+    if (over != 0.0) return;
+    const double rr = cg_total(part, ws), q = sqrt(rr) / sqrt(*rr_old), beta = q * q;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *rr_new = rr;
+        // st[3] counts the iterations, so that every batch of iterations is the
+        // same launch sequence (replayed from one graph)
+        const double it = st[3] + 1.0;
+        st[3] = it;
+        const double rel = sqrt(rr) / sqrt(*bb);
+        st[2] = rel;
+        if (rel < rel_tol) {
+            st[0] = 1.0;
+            st[1] = it;
+        }
+    }
+    for (long k = blockIdx.x * (long)CG_TPB + threadIdx.x; k < n; k += (long)CG_BLOCKS * CG_TPB) p[k] = T(1.0) * r[k] + T(beta) * p[k];
 }
 
 // FP64 reduction over interior points: per-block partials in a fixed order
@@ -1262,7 +1314,9 @@ struct Engine : EngineBase {
     // the first call)
     T *sv_s = nullptr, *sv_t1 = nullptr, *sv_t2 = nullptr, *sv_r = nullptr, *sv_p = nullptr, *sv_ap = nullptr,
       *sv_b = nullptr;
-    double *sv_part = nullptr, *sv_sc = nullptr, *sv_w = nullptr;  // sv_w: xy quadrature weights
+    // sv_p: the h field of sv_s (u = v = 0), so that an apply takes p as it is;
+    // sv_w: xy quadrature weights; sv_pap, sv_rr: partial sums of (p, Ap), (r, r)
+    double *sv_part = nullptr, *sv_sc = nullptr, *sv_w = nullptr, *sv_pap = nullptr, *sv_rr = nullptr;
     static constexpr int DOT_BLOCKS = 256;
     static constexpr int CG_BATCH = 8;  // CG iterations between convergence read-backs
     void xy_dot(const T *a, const T *b, double *out)
@@ -1277,9 +1331,9 @@ struct Engine : EngineBase {
     int helm(const T *z, T *az, double dt)
     {
         int rc;
-        HIP_TRY(hipMemcpyAsync(sv_s + 2 * d.F, z, d.F * sizeof(T), hipMemcpyDeviceToDevice, pl->stream));
+        if (z != sv_p) HIP_TRY(hipMemcpyAsync(sv_p, z, d.F * sizeof(T), hipMemcpyDeviceToDevice, pl->stream));
         if ((rc = apply(sv_t1, sv_s)) || (rc = apply(sv_t2, sv_t1))) return rc;
-        k_axpy<T><<<blocks_for(d.F), TPB, 0, pl->stream>>>(d.F, az, T(1.0), z, T(-(dt * dt)), sv_t2 + 2 * d.F, 0);
+        k_cg_ap<T><<<CG_BLOCKS, CG_TPB, 0, pl->stream>>>(d.F, sv_w, sv_p, sv_t2 + 2 * d.F, T(-(dt * dt)), az, sv_pap);
         return SWE_OK;
     }
     // one CG iteration (cg_solver_mod.f90 L48-88); parity: which of the slots
@@ -1291,16 +1345,13 @@ struct Engine : EngineBase {
         const int a = parity ? 2 : 0, b = parity ? 0 : 2;
         int rc;
         if ((rc = helm(sv_p, sv_ap, dt))) return rc;
-        xy_dot(sv_p, sv_ap, sv_sc + 1);
-        k_cg_step<T><<<blocks_for(F), TPB, 0, pl->stream>>>(F, x, sv_r, sv_p, sv_ap, sv_sc + a, sv_sc + 1, cst);
-        xy_dot(sv_r, sv_r, sv_sc + b);
-        k_cg_check<<<1, 64, 0, pl->stream>>>(sv_sc + b, sv_sc + 3, rel_tol, cst);
-        k_cg_dir<T><<<blocks_for(F), TPB, 0, pl->stream>>>(F, sv_p, sv_r, sv_sc + b, sv_sc + a, cst);
+        k_cg_step<T><<<CG_BLOCKS, CG_TPB, 0, pl->stream>>>(F, sv_w, x, sv_r, sv_p, sv_ap, sv_sc + a, sv_pap, cst, sv_rr);
+        k_cg_dir<T><<<CG_BLOCKS, CG_TPB, 0, pl->stream>>>(F, sv_p, sv_r, sv_rr, sv_sc + a, sv_sc + b, sv_sc + 3, rel_tol, cst);
         return SWE_OK;
     }
     // CG_BATCH iterations (an even number: the slots are back in place
     // after it) from a graph captured for the last (x, dt, rel_tol); the
-    // iterations launch about a dozen small kernels each, whose launch gaps
+    // iterations launch seven small kernels each, whose launch gaps
     // bound the solve at small N
     hipGraphExec_t cg_graph = nullptr;
     const void *cg_key = nullptr;
@@ -1342,10 +1393,13 @@ struct Engine : EngineBase {
             T **st3[] = {&sv_s, &sv_t1, &sv_t2};
             for (T **q : st3)
                 if ((rc = alloc((void **)q, 3 * d.F * sizeof(T)))) return rc;
-            T **f1[] = {&sv_r, &sv_p, &sv_ap, &sv_b};
+            T **f1[] = {&sv_r, &sv_ap, &sv_b};
             for (T **q : f1)
                 if ((rc = field(q))) return rc;
+            sv_p = sv_s + 2 * d.F;
             if ((rc = alloc((void **)&sv_part, DOT_BLOCKS * sizeof(double))) ||
+                (rc = alloc((void **)&sv_pap, CG_BLOCKS * sizeof(double))) ||
+                (rc = alloc((void **)&sv_rr, CG_BLOCKS * sizeof(double))) ||
                 (rc = alloc((void **)&sv_sc, 8 * sizeof(double))) ||
                 (rc = alloc((void **)&sv_w, d.F * sizeof(double))))
                 return rc;
@@ -1374,7 +1428,7 @@ struct Engine : EngineBase {
         int it = 0;
         if (!(rel < rel_tol)) {
             HIP_TRY(hipMemcpyAsync(sv_p, sv_r, F * sizeof(T), hipMemcpyDeviceToDevice, pl->stream));
-            double *cst = sv_sc + 4;  // convergence state (k_cg_check)
+            double *cst = sv_sc + 4;  // convergence state (k_cg_dir)
             k_fill<<<1, 64, 0, pl->stream>>>(cst, 4, 0.0);
             bool done = false;
             it = max_iter + 1;  // not converged (also when max_iter is 0)
