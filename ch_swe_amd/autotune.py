@@ -7,9 +7,9 @@ points that the full 32 x TY tiles leave are split between the two edge
 tiles of an axis) and for both block orders (XCD-aware and plain), keeps the
 fastest, and stores it in a JSON table that create_linear_swm_operator reads
 (ch_swe_amd/tuning.json unless CH_SWE_TUNING names another file).  The
-choices change results only at the level of rounding (a point may move
-between the inner and the edge path of the kernel, which round
-differently).
+stage kernel marches column strips and no longer has tiles, so of the
+candidates only the block order changes the step; the widths shape the
+tiles of the integral diagnostics.
 
     python -m ch_swe_amd.autotune 96 384 --order 42 --precision fp32 [--out FILE]
 

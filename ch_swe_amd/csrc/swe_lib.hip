@@ -132,6 +132,19 @@ __global__ void k_gather(const GatherEntry *__restrict__ e, int n, FieldSet fs)
     dst[g.dst] = T(g.sign) * src[g.src];
 }
 
+// two independent gathers in one launch (2.9 us and a gap each at N = 96)
+template <typename T>
+__global__ void k_gather2(const GatherEntry *__restrict__ e0, int n0, FieldSet f0, const GatherEntry *__restrict__ e1,
+                          int n1, FieldSet f1)
+{
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n0 + n1) return;
+    const GatherEntry g = k < n0 ? e0[k] : e1[k - n0];
+    T *dst = (T *)(k < n0 ? f0.f[g.fields & 15] : f1.f[g.fields & 15]);
+    const T *src = (const T *)(k < n0 ? f0.f[(g.fields >> 4) & 15] : f1.f[(g.fields >> 4) & 15]);
+    dst[g.dst] = T(g.sign) * src[g.src];
+}
+
 template <typename T, int O>
 __global__ void k_xy_cd(Dims d, const T *__restrict__ ut, const T *__restrict__ vt, const T *__restrict__ Jut,
                         const T *__restrict__ Jvt, const T *__restrict__ fJ2, const T *__restrict__ iJa,
@@ -220,10 +233,38 @@ __global__ void k_edge_sync(Dims d, T *__restrict__ up, T *__restrict__ vp, T *_
 #undef D
 }
 
-template <typename T, int O>
+// What an RK4 stage does with its tendency k (rk4_mod.f90 L28-40), as the
+// state assignments would: M 0 out = k; 1 also y = v0 + a k; 2 the step's end
+// v0 = (v0 + b1 k1 + b2 k2) + b2 k3 + b1 k (k not kept).  Passes of their own
+// cost 4.7 us each at N = 96, five a step.
+template <typename T>
+struct RkStage {
+    T *v0, *y;
+    const T *k1, *k2, *k3;
+    T a, b1, b2;
+};
+template <typename T, int M>
+__device__ __forceinline__ void rk_put(const RkStage<T> &r, T *out, long o, T k)
+{
+    if (M < 2) out[o] = k;
+    if (M == 1) {
+        T y = T(1.0) * r.v0[o];
+        y += r.a * k;
+        r.y[o] = y;
+    }
+    if (M == 2) {
+        T x = r.b1 * r.k1[o];
+        x += r.b2 * r.k2[o];
+        T z = r.b2 * r.k3[o];
+        z += r.b1 * k;
+        r.v0[o] = (r.v0[o] + x) + z;
+    }
+}
+
+template <typename T, int O, int M>
 __global__ void k_tend(Dims d, const T *__restrict__ h, const T *__restrict__ up, const T *__restrict__ vp,
                        const T *__restrict__ div, const T *__restrict__ iJu, const T *__restrict__ iJv, T g_hxa,
-                       T H0, T *__restrict__ du, T *__restrict__ dv, T *__restrict__ dh)
+                       T H0, T *__restrict__ out, RkStage<T> rk)
 {
     const int N = d.N;
     const long nu = 6L * N * (N + 1), nh = 6L * (N + 1) * (N + 1);
@@ -232,17 +273,17 @@ __global__ void k_tend(Dims d, const T *__restrict__ h, const T *__restrict__ up
     if (n < nu) {
         unflat(n, N, N + 1, p, i, j);
         long o = off(d, p, i, j);
-        du[o] = -g_hxa * swe::d_i2c_pt<O, T>(swe::line(h + off(d, p, 0, j), 1), 0, N, i) +
-                swe::i_i2c_pt<O, T>(swe::line(up + off(d, p, 0, j), 1), 0, N, i) * iJu[o];
+        rk_put<T, M>(rk, out, o, -g_hxa * swe::d_i2c_pt<O, T>(swe::line(h + off(d, p, 0, j), 1), 0, N, i) +
+                                     swe::i_i2c_pt<O, T>(swe::line(up + off(d, p, 0, j), 1), 0, N, i) * iJu[o]);
     } else if (n < 2 * nu) {
         unflat(n - nu, N + 1, N, p, i, j);
         long o = off(d, p, i, j);
-        dv[o] = -g_hxa * swe::d_i2c_pt<O, T>(swe::line(h + off(d, p, i, 0), d.P), 0, N, j) +
-                swe::i_i2c_pt<O, T>(swe::line(vp + off(d, p, i, 0), d.P), 0, N, j) * iJv[o];
+        rk_put<T, M>(rk, out, d.F + o, -g_hxa * swe::d_i2c_pt<O, T>(swe::line(h + off(d, p, i, 0), d.P), 0, N, j) +
+                                           swe::i_i2c_pt<O, T>(swe::line(vp + off(d, p, i, 0), d.P), 0, N, j) * iJv[o]);
     } else if (n < 2 * nu + nh) {
         unflat(n - 2 * nu, N + 1, N + 1, p, i, j);
         long o = off(d, p, i, j);
-        dh[o] = -H0 * div[o];
+        rk_put<T, M>(rk, out, 2 * d.F + o, -H0 * div[o]);
     }
 }
 
@@ -720,6 +761,7 @@ struct EngineBase {
     KernelTimer timer;
     virtual ~EngineBase() = default;
     virtual int apply(void *out, void *in) = 0;
+    virtual int mk_step(void *v0, void *const k[3], void *const y[2], double dt) = 0;
     virtual int axpy(void *out, double s1, void *x, double s2, void *y, int update) = 0;
     // part: >= 3 INT_MAX_BLOCKS doubles of partial sums, red: 4 doubles (device)
     virtual int integrals(void *st, double *part, double *red, double *mass, double *energy) = 0;
@@ -1099,27 +1141,53 @@ struct Engine : EngineBase {
         k_gather<T><<<blocks_for(n), TPB, 0, pl->stream>>>(m, n, fs);
     }
 
-    template <int O>
-    void apply_o(T *out, T *in)
+    void gather2(const GatherEntry *m0, int n0, T *a0, T *b0, const GatherEntry *m1, int n1, T *a1, T *b1)
+    {
+        k_gather2<T><<<blocks_for(n0 + n1), TPB, 0, pl->stream>>>(m0, n0, FieldSet{{a0, b0, nullptr, nullptr}}, m1, n1,
+                                                                  FieldSet{{a1, b1, nullptr, nullptr}});
+    }
+
+    template <int O, int M>
+    void apply_o(T *out, T *in, const RkStage<T> &rk)
     {
         const int N = d.N;
         T *u = in, *v = in + d.F, *h = in + 2 * d.F;
-        T *du = out, *dv = out + d.F, *dh = out + 2 * d.F;
         long nxy = 6L * (N + 1) * (N + 1), nuv = 6L * N * (N + 1);
         hipStream_t s = pl->stream;
-        gather(maps.xy, maps.n_xy, h, h);
         k_xy_w<T, O><<<blocks_for(nxy), TPB, 0, s>>>(d, u, v, JQ12, W1, W2);
         k_contra<T, O><<<blocks_for(2 * nuv), TPB, 0, s>>>(d, u, v, W1, W2, Qu, iJu, Ju, Qv, iJv, Jv, ut, vt, Jut,
                                                            Jvt);
-        gather(maps.ch, maps.n_ch, Jut, Jvt);
+        gather2(maps.xy, maps.n_xy, h, h, maps.ch, maps.n_ch, Jut, Jvt);
         k_xy_cd<T, O><<<blocks_for(nxy), TPB, 0, s>>>(d, ut, vt, Jut, Jvt, fJ2, iJa, up, vp, div);
-        gather(maps.xyv, maps.n_xyv, up, vp);
-        gather(maps.xy, maps.n_xy, div, div);
+        gather2(maps.xyv, maps.n_xyv, up, vp, maps.xy, maps.n_xy, div, div);
         k_edge_sync<T><<<blocks_for(24L * N), TPB, 0, s>>>(d, up, vp, div, qb, qt, ql, qr);
         const swe_config &c = pl->cfg;
         T g_hxa = T(c.grav / (0.5 * PI / N * c.radius));
-        k_tend<T, O><<<blocks_for(2 * nuv + nxy), TPB, 0, s>>>(d, h, up, vp, div, iJu, iJv, g_hxa, T(c.h_mean), du,
-                                                               dv, dh);
+        k_tend<T, O, M><<<blocks_for(2 * nuv + nxy), TPB, 0, s>>>(d, h, up, vp, div, iJu, iJv, g_hxa, T(c.h_mean), out, rk);
+    }
+    template <int M>
+    void mk_apply(T *out, T *in, const RkStage<T> &rk)
+    {
+        if (order == 21) apply_o<21, M>(out, in, rk);
+        else if (order == 42) apply_o<42, M>(out, in, rk);
+        else apply_o<63, M>(out, in, rk);
+    }
+    // one RK4 step of v0 on the multi-kernel path: registers k1..k3 and two
+    // stage states in turn (a stage's input is read while its output is written)
+    int mk_step(void *v0, void *const k[3], void *const y[2], double dt) override
+    {
+        RkStage<T> rk{(T *)v0, nullptr, (const T *)k[0], (const T *)k[1], (const T *)k[2], T(0), T(dt / 6.0), T(dt / 3.0)};
+        const double A[3] = {0.5 * dt, 0.5 * dt, dt};
+        T *in = (T *)v0;
+        for (int st = 0; st < 3; st++) {
+            rk.y = (T *)y[st & 1];
+            rk.a = T(A[st]);
+            mk_apply<1>((T *)k[st], in, rk);
+            in = rk.y;
+        }
+        mk_apply<2>(nullptr, in, rk);
+        HIP_TRY(hipGetLastError());
+        return SWE_OK;
     }
 
     int apply(void *out, void *in) override
@@ -1127,9 +1195,7 @@ struct Engine : EngineBase {
         if (use_fused) {
             if (order == 21) fused_apply<21>((T *)out, (const T *)in);
             else fused_apply<42>((T *)out, (const T *)in);
-        } else if (order == 21) apply_o<21>((T *)out, (T *)in);
-        else if (order == 42) apply_o<42>((T *)out, (T *)in);
-        else apply_o<63>((T *)out, (T *)in);
+        } else mk_apply<0>((T *)out, (T *)in, RkStage<T>{});
         HIP_TRY(hipGetLastError());
         return SWE_OK;
     }
@@ -1855,28 +1921,17 @@ int swe_rk4_steps(swe_plan *plan, swe_state *v0, double dt, int nsteps)
     if (!std::isfinite(dt)) return fail(SWE_EINVAL, "dt is not finite");
     if (nsteps == 0) return SWE_OK;
     // the RK4 registers are made on first use: the fused path keeps three
-    // (the increment accumulator and two stage states), the unfused one the
-    // reference's five (k1..k4, y)
+    // (the increment accumulator and two stage states), the unfused one five
+    // (k1..k3 and two stage states)
     const int nreg = plan->eng->fused() ? 3 : 5;
     for (int k = 0; k < nreg; k++)
         if (!plan->rk[k] && (rc = swe_state_create(plan, &plan->rk[k]))) return rc;
-    swe_state *k1 = plan->rk[0], *k2 = plan->rk[1], *k3 = plan->rk[2], *k4 = plan->rk[3], *y = plan->rk[4];
-    if (plan->eng->fused()) return plan->eng->rk4(v0->buf, k1->buf, k2->buf, k3->buf, dt, nsteps);
-    // rk4_mod.f90 step_rk4 L28-40: about 45 launches a step on the
-    // multi-kernel path, so chunks of MK_GRAPH_STEPS steps are replayed from a
-    // captured graph (no memset nodes); the rest and timed runs launch directly
-    auto step = [&]() -> int {
-        int r;
-        if ((r = swe_apply(plan, k1, v0))) return r;
-        if ((r = swe_assign(plan, y, 1.0, v0, 0.5 * dt, k1))) return r;
-        if ((r = swe_apply(plan, k2, y))) return r;
-        if ((r = swe_assign(plan, y, 1.0, v0, 0.5 * dt, k2))) return r;
-        if ((r = swe_apply(plan, k3, y))) return r;
-        if ((r = swe_assign(plan, y, 1.0, v0, dt, k3))) return r;
-        if ((r = swe_apply(plan, k4, y))) return r;
-        if ((r = swe_update(plan, v0, dt / 6.0, k1, dt / 3.0, k2))) return r;
-        return swe_update(plan, v0, dt / 3.0, k3, dt / 6.0, k4);
-    };
+    if (plan->eng->fused()) return plan->eng->rk4(v0->buf, plan->rk[0]->buf, plan->rk[1]->buf, plan->rk[2]->buf, dt, nsteps);
+    // rk4_mod.f90 step_rk4 L28-40: 28 launches a step on the multi-kernel path,
+    // so chunks of MK_GRAPH_STEPS steps are replayed from a captured graph (no
+    // memset nodes); the rest and timed runs launch directly
+    void *const ks[3] = {plan->rk[0]->buf, plan->rk[1]->buf, plan->rk[2]->buf}, *const ys[2] = {plan->rk[3]->buf, plan->rk[4]->buf};
+    auto step = [&]() -> int { return plan->eng->mk_step(v0->buf, ks, ys, dt); };
     constexpr int MK_GRAPH_STEPS = 16;
     int done = 0;
     if (!plan->eng->timer.on && nsteps >= MK_GRAPH_STEPS) {
