@@ -12,7 +12,7 @@ import pytest
 
 from test_emu_kernels import emu_exe  # noqa: F401  (fixture)
 
-EDGES = [(10, 42, 64), (11, 42, 64), (13, 21, 32), (63, 42, 32), (64, 42, 64), (122, 42, 32)]
+EDGES = [(10, 42, 64), (11, 42, 64), (13, 21, 32), (63, 42, 32), (64, 42, 64), (122, 42, 32), (176, 21, 32)]
 
 
 @pytest.mark.parametrize("N,order,prec", EDGES)
@@ -27,7 +27,8 @@ def test_strip_edges_under_asan(emu_exe, N, order, prec):  # noqa: F811
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,order,prec", [(11, 42, 64), (63, 21, 64), (64, 42, 64), (121, 42, 64), (122, 42, 64),
-                                          (191, 42, 64), (200, 42, 64), (256, 21, 64), (260, 42, 32)])
+                                          (173, 42, 64), (174, 42, 64), (178, 42, 64), (191, 42, 64), (200, 42, 64),
+                                          (235, 42, 64), (236, 21, 64), (256, 21, 64), (260, 42, 32)])
 def test_strip_edges_match_oracle(oracle_mod, N, order, prec):
     import ch_swe_amd as cs
     from oracle.swe_oracle import MESH_U, MESH_V, MESH_XY
