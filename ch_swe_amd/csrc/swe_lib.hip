@@ -508,6 +508,7 @@ __global__ void k_reduce_final(const double *part, int nb, double *out)
 
 #include "swe_fused.inc"
 #include "swe_fused_host.hpp"
+#include "swe_tiles.inc"
 #include "swe_latlon.inc"
 
 // ---- diagnostics on the multi-kernel path (any SBP order) -------------------
@@ -841,6 +842,9 @@ struct Engine : EngineBase {
     Coef<T> cf{};
     T *rec[2] = {nullptr, nullptr};
     int ntx = 0, nty = 0, ntiles = 0, nseg = 0, fwx = 0, fwy = 0;
+    // FP32: what a single application's kernels (swe_tiles.inc) take besides
+    tiles::Coef<T> tcf{};
+    T *trec = nullptr;
 
     size_t elem() const override { return sizeof(T); }
     bool fused() const override { return use_fused; }
@@ -982,6 +986,15 @@ struct Engine : EngineBase {
         cf = Coef<T>{tabs[0], tabs[1], tabs[2], tabs[3], tabs[4], tabs[5], tabs[6], tabs[7], tf, qb, qt, ql, qr};
         for (auto &r : rec)
             if ((rc = alloc((void **)&r, (size_t)24 * REC_KINDS * n * sizeof(T)))) return rc;
+        if constexpr (sizeof(T) == 4) {
+            T *q[4] = {};
+            for (T *&t : q)
+                if ((rc = alloc((void **)&t, (size_t)n * n * sizeof(T)))) return rc;
+            if ((rc = alloc((void **)&trec, (size_t)24 * tiles::REC_KINDS * n * sizeof(T)))) return rc;
+            tiles::k_coef<T><<<blocks_for((long)n * n), TPB, 0, pl->stream>>>(N, g, q[0], q[1], q[2], q[3]);
+            HIP_TRY(hipGetLastError());
+            tcf = tiles::Coef<T>{tabs[0], tabs[1], q[0], tabs[3], q[1], q[2], tabs[6], q[3], tf, qb, qt, ql, qr};
+        }
         // the kernels' packed cube side table must match the topology
         for (int q = 0; q < 6; q++)
             for (int sdi = 0; sdi < 4; sdi++) {
@@ -1041,6 +1054,27 @@ struct Engine : EngineBase {
     template <int O>
     void fused_apply(T *out, const T *in)
     {
+        if constexpr (sizeof(T) == 4) {
+            timer.launch(tiles::k_records<T, O, TY>, tiles::segments(d.N), tiles::F_REC_THREADS, pl->stream, 1, d, tcf, in, trec);
+            const StageArgs<T> b = stage_args<O>(in);
+            tiles::StageArgs<T> a{};
+            a.d = d;
+            a.c = tcf;
+            a.y = in;
+            a.out = out;
+            a.g_hxa = b.g_hxa;
+            a.H0 = b.H0;
+            a.rec_in = trec;
+            a.ntx = ntx;
+            a.nty = nty;
+            a.fwx = fwx;
+            a.fwy = fwy;
+            a.order = O;
+            a.xcd = b.xcd;
+            a.general = b.general;
+            timer.launch(tiles::k_stage<T, O, TY, 0>, ntiles, tiles::F_THREADS, pl->stream, 0, a);
+            return;
+        }
         launch_records<O>(in, rec[0]);
         StageArgs<T> a = stage_args<O>(in);
         a.out = out;
