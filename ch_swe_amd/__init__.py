@@ -407,11 +407,11 @@ def create_linear_swm_operator(N, order=42, precision=FP64, grav=9.81, h_mean=10
     ensembles and the server take sbp21 / sbp42 plans only);
     linear_blocks=True
     the plain block order of the fused stage kernel; general_tiles=True is
-    accepted (the stage kernel has one path); block_threads (0 or 512) the
+    for the tiles of a single FP32 application; block_threads (0 or 512) the
     fused diagnostics' workgroup size; compensated=True runs RK4 with compensated summation of
     each step's state update (states carry a compensation field); tile_x0 /
-    tile_y0 the first-tile widths of the diagnostics' tiling (0: the library's
-    split; the stage kernel marches column strips and has no tiles).  tuned=True takes the tiling and block order the
+    tile_y0 the first-tile widths of the tilings (diagnostics and single FP32
+    applications; 0: the library's split; RK4 marches column strips).  tuned=True takes the tiling and block order the
     autotuner stored for (N, order, precision) (ch_swe_amd/autotune.py) when
     none is given; results depend on them only at the level of rounding."""
     if tuned and not unfused and not linear_blocks and tile_x0 == 0 and tile_y0 == 0:

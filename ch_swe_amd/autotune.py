@@ -9,7 +9,7 @@ fastest, and stores it in a JSON table that create_linear_swm_operator reads
 (ch_swe_amd/tuning.json unless CH_SWE_TUNING names another file).  The
 stage kernel marches column strips and no longer has tiles, so of the
 candidates only the block order changes the step; the widths shape the
-tiles of the integral diagnostics.
+tiles of the diagnostics and of single FP32 applications.
 
     python -m ch_swe_amd.autotune 96 384 --order 42 --precision fp32 [--out FILE]
 

@@ -39,7 +39,7 @@ enum { SWE_FP64 = 0, SWE_FP32 = 1 };
 enum {
     SWE_FLAG_UNFUSED = 1,      /* run the unfused multi-kernel path (diagnostics) */
     SWE_FLAG_LINEAR_BLOCKS = 2, /* plain block order instead of the XCD-aware one */
-    SWE_FLAG_GENERAL_TILES = 4, /* accepted; the stage kernel has one path for all points */
+    SWE_FLAG_GENERAL_TILES = 4, /* diagnostic: every tile of a single FP32 application takes the general path */
     SWE_FLAG_COMPENSATED = 8    /* RK4 with compensated (Kahan) summation of each step's update of the
                                    state: states carry a compensation field (twice the device memory) */
 };
@@ -69,7 +69,7 @@ typedef struct {
     double axis[3];     /* rotation axis */
     int flags;          /* SWE_FLAG_* bits */
     int block_threads;  /* workgroup size of the fused diagnostics: 0 or 512 (both mean 512) */
-    int tile_x0;        /* width of the first tile along x / y of the fused diagnostics' tiling: */
+    int tile_x0;        /* width of the first tile along x / y of the tilings (diagnostics, FP32 apply): */
     int tile_y0;        /*   0 = the library's split; else 8 .. (what the axis leaves) - 9, within the
                              tile limits (ch_swe_amd/autotune.py sweeps these) */
 } swe_config;
